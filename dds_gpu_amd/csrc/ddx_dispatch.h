@@ -1,0 +1,65 @@
+// Which configurations a batch handle accepts and which kernel runs a batch: host logic only, without
+// HIP, so that it can be checked on the CPU over every configuration.
+#pragma once
+#include "ddx.h"
+
+namespace ddx {
+
+constexpr int kTeamLanes = 16;  // lanes per search of a team
+
+inline bool gpu_config_ok(const ddx_gpu_config& c, int min_log2, int max_log2) {
+  if (c.tt_log2 < min_log2 || c.tt_log2 > max_log2 || (c.jobs_per_deal != 5 && c.jobs_per_deal != 20) ||
+      c.seed_mode < 0 || c.seed_mode > 3)
+    return false;
+  if (c.block < 64 || c.block > 256 || c.block % 64 || c.lanes < 64 || c.lanes % 64 || c.lanes % c.block) return false;
+  if ((c.team != 1 && c.team != kTeamLanes) || c.schedule < 0 || c.schedule > 3) return false;
+  if (c.schedule == DDX_SCHED_THREAD && c.profile) return false;
+  const bool split_schedule = c.schedule == DDX_SCHED_SPLIT && !c.profile;
+  if (c.waves_per_simd != 0 && (c.waves_per_simd < 3 || c.waves_per_simd > 4 || !split_schedule)) return false;
+  if (c.lds_lines != 0 && (c.lds_lines != 3 || c.team != 1 || !split_schedule || c.waves_per_simd == 4)) return false;
+  if (c.split_min_nodes < 0) return false;
+  return c.split_min_nodes == 0 || (c.team == 1 && split_schedule && !c.lds_lines && c.waves_per_simd != 4);
+}
+
+enum class BatchKernel {
+  kNone,      // nothing to solve
+  kWave,      // one wave per search (ddx_wave.hip)
+  kSplit,     // the lane kernels (ddx_gpu.hip): splitting of the tail,
+  kLds,       // the LDS cache of tag lines,
+  kHeld,      // held to waves_per_simd waves,
+  kSchedule,  // or by schedule, profile and, with a profile, team
+};
+struct Dispatch {
+  BatchKernel kernel;
+  long long searches;  // the kernel uses this many of the handle's TTs, stacks and generations
+};
+
+// Batches run with one wave per search, but for those that keep very many lanes busy for long:
+// measured on full deals, 65,536 lanes enter 1.86e9 nodes/s and the wave kernel 3.3e9, but 196,608
+// lanes 3.8e9 while their job queue lasts. A queue shorter than two jobs per lane is mostly tail:
+// 327,680 jobs (8-card endings) on 196,608 lanes take 820 ms with lanes, 380 ms with waves. The
+// measuring options (stage profile, LDS line cache, splitting) exist in the lane kernels only.
+// A handle of at most 1,024 lanes with a long queue (over eight jobs per lane) also stays with
+// the 16 waves that its lanes fill: it is a solver in a corner of the device, and a wave per search
+// would take 64 times as much of it. (The test of stop requests counts on such a batch still
+// running after 1.5 s; the wave kernel would be done with it.)
+//
+// wave_cap: waves of the wave kernel that the device holds at once; 0 in builds without it.
+inline Dispatch dispatch(const ddx_gpu_config& c, int wave_cap, long long jobs) {
+  if (jobs <= 0) return {BatchKernel::kNone, 0};
+  const bool measuring = c.profile || c.lds_lines || c.split_min_nodes > 0;
+  const bool saturated = c.team == 1 && c.lanes > 65536 && jobs > 2 * c.lanes;
+  const bool corner = c.team == 1 && c.lanes <= 1024 && jobs > 8 * c.lanes;
+  if (wave_cap > 0 && !measuring && !saturated && !corner) {
+    long long s = c.lanes / c.team;
+    if (s > wave_cap) s = wave_cap;
+    return {BatchKernel::kWave, s < jobs ? s : jobs};
+  }
+  if (c.split_min_nodes > 0) return {BatchKernel::kSplit, c.lanes};
+  if (c.lds_lines) return {BatchKernel::kLds, c.lanes};
+  if (c.waves_per_simd) return {BatchKernel::kHeld, c.lanes};
+  // Teams have a lane kernel only for the stage profile.
+  return {BatchKernel::kSchedule, c.profile ? c.lanes / c.team : c.lanes};
+}
+
+}  // namespace ddx
