@@ -1,5 +1,5 @@
-// Which configurations a batch handle accepts and which kernel runs a batch: host logic only, without
-// HIP, so that it can be checked on the CPU over every configuration.
+// Which configurations a batch handle accepts, which kernel runs a batch, and the grid of a stream:
+// host logic only, without HIP, so that it can be checked on the CPU over every configuration.
 #pragma once
 #include "ddx.h"
 
@@ -60,6 +60,25 @@ inline Dispatch dispatch(const ddx_gpu_config& c, int wave_cap, long long jobs) 
   if (c.waves_per_simd) return {BatchKernel::kHeld, c.lanes};
   // Teams have a lane kernel only for the stage profile.
   return {BatchKernel::kSchedule, c.profile ? c.lanes / c.team : c.lanes};
+}
+
+// The wave-per-search stream kernel stays on the device until the stream is closed, and the net's
+// kernels, whose seeds the stream may wait for, have to start meanwhile. A SIMD has 512 VGPRs and a
+// wave of the stream takes 80. So a stream has at most 16 waves per CU, and they come in one block
+// per CU, two of which no CU can hold: every SIMD has four waves of it and 192 VGPRs left, in which
+// the net's small kernels (ddx_mlp.hip) find room on every CU. (The node rate of 4 and 6 waves per
+// SIMD differs by 10%.) Fewer searches make smaller blocks, so that they still spread over the CUs.
+constexpr int kStreamWavesPerCu = 16, kStreamVgprs = 80, kSimdVgprs = 512;
+constexpr int kRoomVgprs = kSimdVgprs - kStreamWavesPerCu / 4 * kStreamVgprs;  // per SIMD, beside a stream
+
+struct StreamGrid {
+  long long searches;
+  int blocks, waves;  // waves per block; the last block may hold fewer searches
+};
+inline StreamGrid stream_grid(long long asked, int cus) {
+  const long long most = (long long)kStreamWavesPerCu * cus, n = asked < most ? asked : most;
+  const int waves = (int)((n + cus - 1) / cus);
+  return {n, (int)((n + waves - 1) / waves), waves};
 }
 
 }  // namespace ddx

@@ -18,8 +18,19 @@
 #include "ddx/machine.hpp"
 #include "ddx/pgx.hpp"
 #include "ddx_internal.h"
+#include "ddx_resident.h"
 
 using namespace ddx;
+
+namespace ddx {
+// As g++ compiles it, the static of an inline function has one address per process, in however many
+// of libddx.so, libddx_sig.so and libddx_shared.so it stands. (Never destroyed: handles may outlive it.)
+inline Resident& resident_of_process() {
+  static Resident* r = new Resident;
+  return *r;
+}
+Resident& resident() { return resident_of_process(); }
+}  // namespace ddx
 
 static thread_local std::string g_err;
 

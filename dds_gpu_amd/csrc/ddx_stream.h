@@ -1,6 +1,7 @@
 // The streaming kernels' shared arguments, and the wave-per-search stream kernel's launch
 // (ddx_stream_wave.hip).
 #pragma once
+#include "ddx_dispatch.h"
 #include "ddx_lanes.hpp"
 
 namespace ddx {
@@ -28,9 +29,9 @@ struct StreamArgs {
                                  // [0] produced, [1] end flags (1 = eof, 2 = stop)
 };
 
-// Searches (waves) the wave-per-search stream kernel runs at once, at most; 0 in the builds that
+// The wave-per-search stream kernel's grid for this many searches; no searches in the builds that
 // have no such kernel (signature entries, shared TT).
-int stream_wave_capacity(int device, int* waves);
-int launch_stream_wave(const StreamArgs& a, long long searches, hipStream_t s);
+int stream_wave_grid(int device, long long asked, StreamGrid* g);
+int launch_stream_wave(const StreamArgs& a, const StreamGrid& g, hipStream_t s);
 
 }  // namespace ddx

@@ -24,6 +24,7 @@
 #include <new>
 #include <vector>
 
+#include "ddx_resident.h"
 #include "ddx_stream.h"
 
 using namespace ddx;
@@ -195,7 +196,9 @@ static T* dev_ptr(T* host) {
   return (T*)d;
 }
 
+// The kernel is not running (any more).
 static void stream_free(ddx_stream* s) {
+  count_stream(s->cfg.device, -1);
   lanes_free(s->lanes);
   if (s->hands) (void)hipHostFree(s->hands);
   if (s->seeds) (void)hipHostFree(s->seeds);
@@ -245,16 +248,16 @@ extern "C" int ddx_stream_open(const ddx_gpu_config* cfg_in, int ring_slots, ddx
   // through 4,096 searches and a ring of 256 took 912 ms with one lane per search, 45 ms now. TTs only
   // for the searches that run: more would lie unused, and memory that others freed has to be
   // cleared by the driver first (10 GB took 250 ms).
-  int waves = 0;
-  int rc = stream_wave_capacity(cfg.device, &waves);
+  StreamGrid waves;
+  int rc = stream_wave_grid(cfg.device, cfg.lanes / cfg.team, &waves);
   if (rc != DDX_OK) {
     delete s;
     return rc;
   }
-  long long searches = cfg.lanes / cfg.team;
-  if (waves && searches > waves) searches = waves;
-  rc = lanes_alloc(s->lanes, searches, cfg.tt_log2);
+  count_stream(cfg.device, 1);  // before lanes_alloc, which synchronizes the device (ddx_resident.h)
+  rc = lanes_alloc(s->lanes, waves.searches ? waves.searches : cfg.lanes, cfg.tt_log2);
   if (rc != DDX_OK) {
+    count_stream(cfg.device, -1);
     delete s;
     return rc;
   }
@@ -301,7 +304,7 @@ extern "C" int ddx_stream_open(const ddx_gpu_config* cfg_in, int ring_slots, ddx
   a.seed_mode = cfg.seed_mode;
   if (!a.hands || !a.seeds || !a.out || !a.work || !a.comp || !a.ctl) return fail("mapped views");
   s->t0 = std::chrono::steady_clock::now();
-  if (waves) rc = launch_stream_wave(a, searches, s->stream);
+  if (waves.searches) rc = launch_stream_wave(a, waves, s->stream);
 #if DDX_TT_SIG || DDX_SHARED_TT
   const dim3 grid((unsigned)(cfg.lanes / 256));
   if (cfg.waves_per_simd == 3) hipLaunchKernelGGL(stream_kernel_w3, grid, dim3(256), 0, s->stream, a);

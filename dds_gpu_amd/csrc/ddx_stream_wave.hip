@@ -25,10 +25,6 @@ using namespace ddx;
 namespace {
 
 constexpr int kPollers = 8;
-// Four waves per SIMD: the persistent kernel must leave registers for other kernels of the
-// process -- the net's predictions run while it does -- and with 4 x 80 of 512 VGPRs taken there
-// are 192 left. (The node rate of 4 and 6 waves per SIMD differs by 10%.)
-constexpr int kWavesPerCu = 16;
 
 template <class V>
 __device__ __forceinline__ V load_sys(const V* p) {
@@ -41,8 +37,9 @@ __device__ __forceinline__ V load_dev(const V* p) {
 
 }  // namespace
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void stream_kernel_wave(StreamArgs a) {
-  const long long search = blockIdx.x;
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6, 6))) void stream_kernel_wave(StreamArgs a) {
+  const long long search = (long long)blockIdx.x * (blockDim.x >> 6) + uni((int)(threadIdx.x >> 6));
+  if (search >= a.lanes.searches) return;  // in the last block (no wave waits for another)
   WaveSearch W;
   W.init(a.lanes, search);
   const int jpd = a.jobs_per_deal;
@@ -116,15 +113,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void
 
 namespace ddx {
 
-int stream_wave_capacity(int device, int* waves) {
+int stream_wave_grid(int device, long long asked, StreamGrid* g) {
   int cus = 0;
   HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  *waves = kWavesPerCu * cus;
+  *g = stream_grid(asked, cus);
   return DDX_OK;
 }
 
-int launch_stream_wave(const StreamArgs& a, long long searches, hipStream_t s) {
-  hipLaunchKernelGGL(stream_kernel_wave, dim3((unsigned)searches), dim3(64), 0, s, a);
+int launch_stream_wave(const StreamArgs& a, const StreamGrid& g, hipStream_t s) {
+  hipLaunchKernelGGL(stream_kernel_wave, dim3((unsigned)g.blocks), dim3(64 * g.waves), 0, s, a);
   HIPCHECK(hipGetLastError());
   return DDX_OK;
 }
@@ -134,11 +131,11 @@ int launch_stream_wave(const StreamArgs& a, long long searches, hipStream_t s) {
 #else
 namespace ddx {
 
-int stream_wave_capacity(int, int* waves) {
-  *waves = 0;
+int stream_wave_grid(int, long long, StreamGrid* g) {
+  *g = {0, 0, 0};
   return DDX_OK;
 }
-int launch_stream_wave(const StreamArgs&, long long, hipStream_t) { return DDX_E_ARG; }
+int launch_stream_wave(const StreamArgs&, const StreamGrid&, hipStream_t) { return DDX_E_ARG; }
 
 }  // namespace ddx
 #endif

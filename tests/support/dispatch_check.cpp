@@ -1,6 +1,7 @@
 // Every configuration that a batch handle accepts, against the storage it allocates (lanes / team
 // TTs, stacks and generations): no batch size may reach a kernel that indexes past them, an empty
-// batch reaches none. Prints the configurations tried, the batches, and the faults.
+// batch reaches none. And the stream's grid: its searches, in at most a block per CU. Prints the
+// configurations tried, the batches, and the faults.
 #include <stdio.h>
 
 #include <initializer_list>
@@ -36,6 +37,15 @@ int main() {
                       }
                     }
                   }
+  for (int cus = 1; cus <= 320; cus++)
+    for (long long n : {1ll, 4ll, 64ll, 255ll, 256ll, 257ll, 2048ll, 4096ll, 65536ll, 196608ll}) {
+      const StreamGrid g = stream_grid(n, cus);
+      const bool covers = (long long)g.blocks * g.waves >= g.searches && (long long)(g.blocks - 1) * g.waves < g.searches;
+      const bool most = g.searches == n || g.searches == 16ll * cus;
+      if (!covers || !most || g.searches < 1 || g.searches > n || g.blocks > cus || g.waves < 1 || g.waves > 16) bad++;
+    }
+  // A full block leaves kRoomVgprs on every SIMD, and no room for a second one.
+  if (kRoomVgprs != 512 - 4 * kStreamVgprs || 8 * kStreamVgprs <= 512) bad++;
   printf("%ld %ld %ld\n", configs, batches, bad);
   return bad != 0;
 }
