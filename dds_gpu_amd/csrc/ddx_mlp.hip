@@ -826,6 +826,7 @@ struct ddx_mlp {
   int cus = 0;
   hipStream_t s = nullptr;
   hipEvent_t used = nullptr;  // the last prediction on a caller's stream
+  std::vector<void*> outgrown;  // buffers to free when no stream is open
 };
 
 constexpr long long kPinDeals = 64;  // deals that ddx_mlp_predict_host passes through mapped memory
@@ -833,14 +834,36 @@ constexpr int kMaxShares = 32;
 
 static long long units_of(long long deals) { return (deals + 15) / 16 * 5; }
 
+// Gives up a buffer that is to be replaced by a larger one. hipFree waits for the whole device, so
+// beside an open stream, whose kernel does not end, the buffer is kept for a later time.
+template <class T>
+static void give_up(ddx_mlp* h, T*& p) {
+  std::lock_guard<std::mutex> lock(ddx::resident().mu);  // no stream opens meanwhile
+  bool keep = ddx::resident().streams(h->device) != 0;
+  if (keep && p) {
+    try {
+      h->outgrown.push_back(p);
+    } catch (const std::bad_alloc&) {
+      keep = false;
+    }
+  }
+  if (!keep) {
+    if (p) (void)hipFree(p);
+    for (void* q : h->outgrown) (void)hipFree(q);
+    h->outgrown.clear();
+  }
+  p = nullptr;
+}
+// The size for a buffer that holds `cap` and has to hold n: few growths, and what is outgrown beside a
+// stream together no more than the buffer.
+static long long grown(long long cap, long long n) { return n < 2 * cap ? 2 * cap : n; }
+
 // Buffers of a training step of `deals` deals (rounded up to 16).
 static int train_reserve(ddx_mlp* h, long long deals, long long steps) {
   const long long units = units_of(deals);
   if (units > h->cap) {
-    if (h->acts) (void)hipFree(h->acts);
-    if (h->x) (void)hipFree(h->x);
-    h->acts = nullptr;
-    h->x = nullptr;
+    give_up(h, h->acts);
+    give_up(h, h->x);
     h->cap = 0;
     HIPCHECK(hipMalloc(&h->acts, (size_t)units * 64 * (4 * H + OUT) * 2));
     HIPCHECK(hipMalloc(&h->x, (size_t)units / 5 * IN * 2));
@@ -848,8 +871,8 @@ static int train_reserve(ddx_mlp* h, long long deals, long long steps) {
   }
   if (!h->parts) HIPCHECK(hipMalloc(&h->parts, (size_t)kMaxShares * NPARAM * 4));
   if (steps > h->stats_cap) {
-    if (h->stats) (void)hipFree(h->stats);
-    h->stats = nullptr;
+    give_up(h, h->stats);
+    steps = grown(h->stats_cap, steps);
     h->stats_cap = 0;
     HIPCHECK(hipMalloc(&h->stats, (size_t)steps * 8));
     h->stats_cap = steps;
@@ -859,14 +882,13 @@ static int train_reserve(ddx_mlp* h, long long deals, long long steps) {
 
 static int mlp_stage_host(ddx_mlp* h, const uint64_t* hands, const uint8_t* tables, long long n) {
   if (n > h->host_cap) {
-    if (h->d_hands) (void)hipFree(h->d_hands);
-    if (h->d_tables) (void)hipFree(h->d_tables);
-    h->d_hands = nullptr;
-    h->d_tables = nullptr;
+    give_up(h, h->d_hands);
+    give_up(h, h->d_tables);
+    const long long cap = grown(h->host_cap, n);
     h->host_cap = 0;
-    HIPCHECK(hipMalloc(&h->d_hands, n * 32));
-    HIPCHECK(hipMalloc(&h->d_tables, n * 20));
-    h->host_cap = n;
+    HIPCHECK(hipMalloc(&h->d_hands, cap * 32));
+    HIPCHECK(hipMalloc(&h->d_tables, cap * 20));
+    h->host_cap = cap;
   }
   HIPCHECK(hipMemcpyAsync(h->d_hands, hands, n * 32, hipMemcpyHostToDevice, h->s));
   if (tables) HIPCHECK(hipMemcpyAsync(h->d_tables, tables, n * 20, hipMemcpyHostToDevice, h->s));
@@ -988,6 +1010,7 @@ extern "C" void ddx_mlp_destroy(ddx_mlp* h) {
                   h->parts, h->stats, h->d_order, h->d_hands, h->d_tables, h->d_seeds};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
+  for (void* q : h->outgrown) (void)hipFree(q);
   if (h->s) (void)hipStreamDestroy(h->s);
   if (h->used) (void)hipEventDestroy(h->used);
   delete h;
@@ -1043,11 +1066,11 @@ extern "C" int ddx_mlp_train(ddx_mlp* h, const uint64_t* hands, const uint8_t* t
   // three kernels and nothing else, and the host waits at the end only.
   if ((rc = mlp_stage_host(h, hands, tables, n)) != DDX_OK) return rc;
   if (n > h->order_cap) {
-    if (h->d_order) (void)hipFree(h->d_order);
-    h->d_order = nullptr;
+    give_up(h, h->d_order);
+    const long long cap = grown(h->order_cap, n);
     h->order_cap = 0;
-    HIPCHECK(hipMalloc(&h->d_order, n * 8));
-    h->order_cap = n;
+    HIPCHECK(hipMalloc(&h->d_order, cap * 8));
+    h->order_cap = cap;
   }
   std::vector<long long> order(n);
   for (long long i = 0; i < n; i++) order[i] = i;
@@ -1143,11 +1166,11 @@ extern "C" int ddx_mlp_predict_host(ddx_mlp* h, const uint64_t* hands, int64_t n
   }
   if ((rc = mlp_stage_host(h, hands, nullptr, n)) != DDX_OK) return rc;
   if (n > h->seeds_cap) {
-    if (h->d_seeds) (void)hipFree(h->d_seeds);
-    h->d_seeds = nullptr;
+    give_up(h, h->d_seeds);
+    const long long cap = grown(h->seeds_cap, n);
     h->seeds_cap = 0;
-    HIPCHECK(hipMalloc(&h->d_seeds, n * 20 + 16));
-    h->seeds_cap = n;
+    HIPCHECK(hipMalloc(&h->d_seeds, cap * 20 + 16));
+    h->seeds_cap = cap;
   }
   launch_predict(h, h->s, h->d_hands, n, h->d_seeds, false);
   HIPCHECK(hipGetLastError());

@@ -76,6 +76,31 @@ def net_case(ddx):
         assert np.array_equal(a, b)
 
 
+def growth_case(ddx):
+    """Calls that outgrow the buffers of earlier ones."""
+    g = np.load(os.path.join(ROOT, "tests", "golden", "full_2000.npz"))
+    hands, tables = g["hands"], g["tables"]
+    nets = [ddx.TrickNet(path=os.path.join(ROOT, "dds_gpu_amd", "models", "tricknet.bin")) for _ in range(2)]
+
+    def first(net):
+        net.predict(hands[:100])
+        net.train(hands[:300], tables[:300], batch_deals=100, lr=1e-4)
+
+    def more(net):
+        out = [timed("predict %d" % n, lambda: net.predict(hands[:n])) for n in (150, 900, 2000)]
+        for n, batch in ((900, 100), (2000, 300)):
+            timed("training on %d" % n, lambda: net.train(hands[:n], tables[:n], batch_deals=batch, lr=1e-4))
+        out.append(net.params())
+        return out + [timed("gradients of 700", lambda: net.grads(hands[:700], tables[:700]))[0]]
+
+    for net in nets:
+        first(net)
+    alone, beside = more(nets[0]), beside_stream(ddx, lambda: more(nets[1]))
+    more(nets[1])  # what was outgrown is freed
+    for a, b in zip(alone, beside):
+        assert np.array_equal(a, b)
+
+
 def batch_case(ddx):
     hands = ddx.random_deals(32, 300, 6)
     want, cpu = ddx.cpu_solve(hands, tt_log2=9)
@@ -86,7 +111,7 @@ def batch_case(ddx):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", ["net", "batch"])
+@pytest.mark.parametrize("case", ["net", "growth", "batch"])
 def test_runs_while_a_stream_is_open(case):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), case], cwd=ROOT, capture_output=True, text=True,
                        timeout=100)
@@ -137,4 +162,4 @@ if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     import torch  # noqa: F401 -- before the ddx library: one HIP runtime for both
     from dds_gpu_amd import ddx as module
-    {"net": net_case, "batch": batch_case}[sys.argv[1]](module)
+    {"net": net_case, "growth": growth_case, "batch": batch_case}[sys.argv[1]](module)
