@@ -991,9 +991,9 @@ extern "C" int ddx_mlp_create(int device, uint64_t seed, ddx_mlp** out) {
   ddx::init_matrix(p.data() + OFF_W1, H, IN, H, IN_USED, IN_USED, rng);
   ddx::init_matrix(p.data() + OFF_W2, H, H, H, H, H, rng);
   ddx::init_matrix(p.data() + OFF_W3, OUT, H, OUT_USED, H, H, rng);
-  HIPCHECK(hipMemcpy(h->p, p.data(), NPARAM * 4, hipMemcpyHostToDevice));
-  HIPCHECK(hipMemset(h->m, 0, NPARAM * 4));
-  HIPCHECK(hipMemset(h->v, 0, NPARAM * 4));
+  HIPCHECK(hipMemcpyAsync(h->p, p.data(), NPARAM * 4, hipMemcpyHostToDevice, h->s));
+  HIPCHECK(hipMemsetAsync(h->m, 0, NPARAM * 4, h->s));
+  HIPCHECK(hipMemsetAsync(h->v, 0, NPARAM * 4, h->s));
   sync_bf16(h);
   HIPCHECK(hipStreamSynchronize(h->s));
   *out = h;
@@ -1021,13 +1021,15 @@ extern "C" int64_t ddx_mlp_param_count(void) { return (int64_t)NPARAM; }
 extern "C" int ddx_mlp_params(ddx_mlp* h, float* buf, int get) {
   if (!h || !buf) return DDX_E_ARG;
   HIPCHECK(hipSetDevice(h->device));
+  // On the handle's stream, behind the predictions that still read the parameters (ddx_mlp_predict).
   if (get) {
-    HIPCHECK(hipMemcpy(buf, h->p, NPARAM * 4, hipMemcpyDeviceToHost));
+    HIPCHECK(hipMemcpyAsync(buf, h->p, NPARAM * 4, hipMemcpyDeviceToHost, h->s));
   } else {
-    HIPCHECK(hipMemcpy(h->p, buf, NPARAM * 4, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpyAsync(h->p, buf, NPARAM * 4, hipMemcpyHostToDevice, h->s));
     sync_bf16(h);
-    HIPCHECK(hipStreamSynchronize(h->s));
+    HIPCHECK(hipGetLastError());
   }
+  HIPCHECK(hipStreamSynchronize(h->s));
   return DDX_OK;
 }
 

@@ -218,14 +218,16 @@ int ddx_mlp_grads(ddx_mlp* h, const uint64_t* hands, const uint8_t* tables, int6
 int ddx_mlp_train(ddx_mlp* h, const uint64_t* hands, const uint8_t* tables, int64_t n, int epochs,
                   int batch_deals, float lr, uint64_t shuffle_seed, float* loss_acc);
 /* Seeds (most likely NS tricks) for n deals: device buffers d_hands[4n] -> d_seeds[20n], ordered
- * on HIP stream `stream` (NULL: synchronous). */
+ * on HIP stream `stream` (NULL: synchronous). Training, new parameters and ddx_mlp_destroy wait for
+ * predictions queued before; those that a graph captured are the caller's to order. */
 int ddx_mlp_predict(ddx_mlp* h, const uint64_t* d_hands, int64_t n, uint8_t* d_seeds, void* stream);
 /* Same with host buffers. */
 int ddx_mlp_predict_host(ddx_mlp* h, const uint64_t* hands, int64_t n, uint8_t* seeds);
 /* ddx_mlp_predict that allocates nothing, for callers that cannot allocate (code under HIP
  * graph capture, tight serving loops). No counterpart in the reference. n is at most 256 deals
  * (DDX_E_ARG beyond). Kernels run on `stream` (NULL: the null stream, and the call returns when
- * the seeds are written). */
+ * the seeds are written). The net keeps no record of these calls: the caller lets them end before
+ * it trains the net, gives it new parameters or destroys it. */
 int ddx_mlp_predict_noalloc(const ddx_mlp* h, const uint64_t* d_hands, int64_t n, uint8_t* d_seeds,
                             void* stream);
 int ddx_mlp_save(ddx_mlp* h, const char* path);
