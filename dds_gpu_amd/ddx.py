@@ -78,6 +78,8 @@ def lib(variant=""):
         L.ddx_gpu_open.argtypes = [P, P]
         L.ddx_gpu_close.argtypes = [P]
         L.ddx_gpu_device_bytes.argtypes = [P]
+        L.ddx_gpu_waves.argtypes = [P, I64]
+        L.ddx_gpu_waves.restype = I64
         L.ddx_gpu_device_bytes.restype = U64
         L.ddx_gpu_solve.argtypes = [P, P, I64, P, P, P]
         L.ddx_gpu_solve_async.argtypes = [P, P, I64, P, P, P]
@@ -255,6 +257,10 @@ class GpuSolver:
     @property
     def device_bytes(self):
         return self._L.ddx_gpu_device_bytes(self.h)
+
+    def waves(self, n):
+        """Searches a batch of n deals runs with, one per wave; 0: a kernel with one lane per search."""
+        return self._L.ddx_gpu_waves(self.h, n)
 
     def progress(self):
         v = ctypes.c_uint64()

@@ -163,6 +163,9 @@ int ddx_gpu_open(const ddx_gpu_config* cfg, ddx_gpu** out);
 void ddx_gpu_close(ddx_gpu* h);
 /* Device bytes held by the handle. */
 uint64_t ddx_gpu_device_bytes(const ddx_gpu* h);
+/* Searches that a batch of n deals runs with, each on a wave of its own; 0 when a kernel with one
+ * lane per search runs it (see above). */
+int64_t ddx_gpu_waves(const ddx_gpu* h, int64_t n);
 
 /* Solves n deals: host hands[4n] in, host out[20n] (0xFF = unsolved after a stop). seeds:
  * host n*20 NS-trick seeds for DDX_SEED_STEP/CERT, else NULL. Replaces the reference's
