@@ -21,8 +21,8 @@ up to ~1e9 nodes), far more than a bench can run to completion, so:
                reference's own measure, README.md:166-176), which decays as heavy jobs pile up
 
 Legs (the same deals and queue order in each):
-  plain    the plain wavefront kernel: 65,536 lanes, one lane per search, TT_LOG2 10 per lane,
-           5 jobs per deal, binary search from 7 (DDX_SEED_PLAIN)
+  plain    the reference's configuration: 65,536 lanes, TT_LOG2 10 per search, 5 jobs per deal,
+           binary search from 7 (DDX_SEED_PLAIN); the exact build runs it with a wave per search
   tuned    the autotuned persistent configuration (dds_gpu_amd/tuned.json), plain seeds
   learned  the tuned configuration seeded by the trick-count net (DDX_SEED_CERT): the net's
            GPU prediction for the whole batch is timed and its cost charged pro rata
@@ -36,7 +36,8 @@ Checks and side measurements in the same JSON line:
                 reference CPU solver's tables (tests/golden/full_2000.npz); a mismatch exits 1
   roofline      the headline leg's solve kernel: algorithmic TT bytes per launch (64 B per probed
                 tag line, 16 B per entry read, 144 B per store, 52 B of deal I/O per finished
-                table) over the kernel's HIP-event duration, against the 8 TB/s HBM peak
+                table) over the kernel's HIP-event duration, against the 8 TB/s HBM peak. (A leg
+                with a wave per search reads whole buckets, 320 B a probe: its tt_bytes_requested)
   cpu_baseline  the reference's own CPU solver (oracle/_ref/dd_cpu, built from the reference
                 sources) on a bounded sample of the same deals, all host cores, TT_LOG2 18
                 (its default); it also re-checks that sample's fixture tables
@@ -61,6 +62,9 @@ HBM_PEAK_GBS = 8000.0
 # stores read and rewrite the 64 B tag line and write one entry; the shared store reads the tag
 # line and writes one 4 B tag and one entry).
 TT_BYTES = {"": (16.0, 144.0), "sig": (12.0, 140.0), "shared": (32.0, 100.0)}
+# A wave's search reads a bucket's tags and entries together: bytes per probe, and per store (the tag
+# line and one entry).
+WAVE_BYTES = (320.0, 80.0)
 PLAIN = {"lanes": 65536, "team": 1, "tt_log2": 10, "jobs_per_deal": 5, "schedule": 2, "waves_per_simd": 0,
          "block": 256}
 DEFAULT_MODEL = os.path.join(ROOT, "dds_gpu_amd", "models", "tricknet.bin")
@@ -159,7 +163,9 @@ def run_leg(ddx, torch, name, cfg, d_hands, n, a, gold, seeds=None, predict_s=0.
                       block=cfg.get("block", 256), variant=cfg.get("variant", ""),
                       seed_mode=ddx.SEED_CERT if seeds is not None else ddx.SEED_PLAIN)
     jpd = cfg["jobs_per_deal"]
-    log("[%s] %s, %.1f GB of lane state" % (name, json.dumps(cfg), g.device_bytes / 1e9))
+    waves = g.waves(n)
+    log("[%s] %s, %.1f GB of lane state, %s" % (name, json.dumps(cfg), g.device_bytes / 1e9,
+                                                "a wave per search, %d at once" % waves if waves else "a lane per search"))
     torch.cuda.synchronize()
     g.solve_async(d_hands.data_ptr(), n, d_out.data_ptr(),
                   d_seeds=seeds.data_ptr() if seeds is not None else 0, stream=stream)
@@ -207,9 +213,11 @@ def run_leg(ddx, torch, name, cfg, d_hands, n, a, gold, seeds=None, predict_s=0.
            "nodes_per_table": round((nd1 - nd0) / max(window_tables, 1e-9), 0),
            "predict_s_charged": round(charge, 5),
            "bit_exact": {"checked_answers": int(solved.sum()), "wrong": wrong},
-           "kernel": {"ms": round(kms, 1), "alg_bytes": alg, "achieved_gbs": round(achieved, 3),
+           "kernel": {"ms": round(kms, 1), "waves": waves, "alg_bytes": alg, "achieved_gbs": round(achieved, 3),
                       "nodes": st.nodes, "tt_probes": st.tt_probes, "tt_entry_reads": st.tt_entry_reads,
                       "tt_stores": st.tt_stores, "jobs_done": st.jobs_done}}
+    if waves:
+        res["kernel"]["tt_bytes_requested"] = WAVE_BYTES[0] * st.tt_probes + WAVE_BYTES[1] * st.tt_stores
     log("[%s] %d whole tables in %.1f s from launch: %.2f tables/s (window rate %.2f); %d answers "
         "checked, %d wrong" % (name, whole, from_launch, value, window_rate, solved.sum(), wrong))
     return res

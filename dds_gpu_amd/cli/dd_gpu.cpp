@@ -7,18 +7,21 @@
 // TT_LOG2 < 9). Environment:
 //   THREADS     solver lanes (default 32768; clamped to the jobs, rounded up to 256)
 //   TIME_LIMIT  seconds; then the lanes stop and unfinished answers are skipped in the check
+// Most batches run with one wave per search, THREADS of them at most; the kernels with one lane per
+// search, which SCHEDULE, CHEAP_LOOP, WAVES, LDS and WAVE are about, take over 65,536 THREADS with more
+// than two jobs each (ddx.h says which else). The second line of the output says what runs.
 //   SCHEDULE    0 priority (the reference's), 1 chain (CHEAP_LOOP=1), 2 split (default)
 //   PER_LEAD=1  one job per lead (20 per deal) instead of per strain
 //   SEEDS=FILE  n x 20 uint8 NS-trick seeds for the seeded search (DDX_SEED_CERT)
 //   MODEL=FILE  a trained trick-count net (dd_train): its predictions seed DDX_SEED_CERT; the
 //               prediction time is counted in the reported time
-//   TEAM=16     sixteen lanes per search (THREADS / 16 searches)
-//   WAVES=3|4   hold the kernel to that many waves per SIMD (split schedule); the tuned
-//               configuration for full deals is THREADS=196608 WAVES=3 with TT_LOG2 11
+//   TEAM=16     THREADS / 16 searches, on waves whatever their number
+//   WAVES=3|4   hold the lane kernel to that many waves per SIMD (split schedule); the tuned
+//               configuration for full deals is THREADS=196608 WAVES=3 with TT_LOG2 12
 //   LDS=3       keep each lane's last 3 TT tag lines in LDS (one lane per search)
-//   WAVE=0      the per-thread kernel: no wave schedule, each lane runs its own next stage
-//               (DDX_SCHED_THREAD; the reference's WAVE=0 solve_kernel). Unset or 1: the
-//               wavefront kernel with SCHEDULE
+//   WAVE=0      the lane kernel without a wave schedule, each lane running its own next stage
+//               (DDX_SCHED_THREAD; the reference's WAVE=0 solve_kernel). Unset or 1: the one
+//               with SCHEDULE
 //   STACK_KB    accepted for compatibility: frames live in HBM, there is no stack limit to set
 #include <stdio.h>
 #include <stdlib.h>
@@ -117,15 +120,17 @@ int main(int argc, char** argv) {
   }
   printf("%lld threads, ", threads);
   printf("%lld deals, %lld solves, TT %.0f KB/solve, %.2f GB total\n", n, jobs,
-         320.0 * (1 << tt_log2) / 1024.0, 320.0 * (double)threads * (1 << tt_log2) / 1e9);
-  if (cfg.schedule == DDX_SCHED_THREAD) printf("per-thread kernel\n");
-  else printf("wavefront kernel, schedule %d\n", cfg.schedule);
+         320.0 * (1 << tt_log2) / 1024.0, 320.0 * (double)(threads / cfg.team) * (1 << tt_log2) / 1e9);
   fflush(stdout);
   ddx_gpu* h = nullptr;
   if (ddx_gpu_open(&cfg, &h) != DDX_OK) {
     fprintf(stderr, "%s\n", ddx_last_error());
     return 1;
   }
+  if (const long long waves = ddx_gpu_waves(h, n)) printf("wavefront kernel, one wave per search, %lld at once\n", waves);
+  else if (cfg.schedule == DDX_SCHED_THREAD) printf("per-thread kernel\n");
+  else printf("wavefront kernel, one lane per search, schedule %d\n", cfg.schedule);
+  fflush(stdout);
   const double limit = getenv("TIME_LIMIT") ? atof(getenv("TIME_LIMIT")) : 1e18;
   std::vector<uint8_t> got(n * 20);
   std::atomic<bool> running{true};

@@ -8,14 +8,15 @@
 //                                    deal (default 50) re-solved on the CPU and compared
 // Same argv, records, stderr lines and exit codes as the reference's gpu/stream_main.cu
 // (0 = no mismatch, 1 = mismatch or GPU error, 2 = usage / TT_LOG2 < 9). Environment:
-//   THREADS      solver lanes (default 32768, rounded up to 256)
+//   THREADS      searches at once (default 32768, rounded up to 256; at most 4096 run, a wave each)
 //   PER_LEAD     0 (default, as the reference): one job per strain; 1: one job per lead,
-//                which keeps four times as many lanes busy when the ring holds few deals
+//                which keeps four times as many searches busy when the ring holds few deals
 //   RING         ring slots (default 4096)
 //   RATE         bench: Poisson arrivals at RATE deals/s (default 0 = as fast as slots free)
 //   SEED         bench: deal stream seed (default 2026)
-//   TEAM=16      sixteen lanes per search (THREADS / 16 searches)
-//   WAVES=3      hold the kernel to 3 waves per SIMD
+//   TEAM=16      THREADS / 16 searches
+//   WAVES=3      bin/sig and bin/shared, which run one lane per search: hold the kernel to 3 waves
+//                per SIMD
 //   MODEL=FILE   a trained trick-count net: each deal's 20 predictions are computed on the GPU
 //                when it arrives (inside its latency) and seed the search (DDX_SEED_CERT)
 // Bench prints the latency from arrival to result, p50 and p99 in ms, over the deals that
@@ -81,14 +82,15 @@ int main(int argc, char** argv) {
   const int ring = getenv("RING") ? atoi(getenv("RING")) : 4096;
   const double rate = getenv("RATE") ? atof(getenv("RATE")) : 0;
   const uint64_t seed = getenv("SEED") ? strtoull(getenv("SEED"), 0, 10) : 2026;
-  fprintf(stderr, "%lld threads (%d per search), TT %.2f GB total, %d jobs per deal, ring %d deals%s\n",
-          (long long)cfg.lanes, cfg.team, 320.0 * cfg.lanes / cfg.team * (1 << tt_log2) / 1e9,
-          cfg.jobs_per_deal, ring, net ? ", learned seeds" : "");
   ddx_stream* s = nullptr;
   if (ddx_stream_open(&cfg, ring, &s) != DDX_OK) {
     fprintf(stderr, "%s\n", ddx_last_error());
     return 1;
   }
+  const long long searches = ddx_stream_searches(s);
+  fprintf(stderr, "%lld threads (%d per search), %lld searches at once, TT %.2f GB total, %d jobs per deal, ring %d deals%s\n",
+          (long long)cfg.lanes, cfg.team, searches, 320.0 * searches * (1 << tt_log2) / 1e9, cfg.jobs_per_deal, ring,
+          net ? ", learned seeds" : "");
   const auto t0 = Clock::now();
   std::mutex mu;
   std::vector<double> arrival;  // by deal id

@@ -326,6 +326,8 @@ extern "C" int ddx_stream_open(const ddx_gpu_config* cfg_in, int ring_slots, ddx
   return DDX_OK;
 }
 
+extern "C" int64_t ddx_stream_searches(const ddx_stream* s) { return s ? s->lanes.lanes : 0; }
+
 extern "C" int ddx_stream_push(ddx_stream* s, const uint64_t hands[4], const uint8_t* seeds20,
                                int64_t id) {
   if (!s || !hands || !ddx_check_deal(hands)) {

@@ -89,6 +89,8 @@ def lib(variant=""):
         L.ddx_gpu_last_kernel_ms.restype = ctypes.c_double
         L.ddx_gpu_profile.argtypes = [P, P, I]
         L.ddx_gpu_progress.argtypes = [P, P]
+        L.ddx_stream_searches.argtypes = [P]
+        L.ddx_stream_searches.restype = I64
         L.ddx_stream_open.argtypes = [P, I, P]
         L.ddx_stream_push.argtypes = [P, P, P, I64]
         L.ddx_stream_poll.argtypes = [P, I, P, P, P]
@@ -339,6 +341,10 @@ class Stream:
                                      ctypes.byref(got)))
         n = got.value
         return self._ids[:n].copy(), self._tab[:n].copy()
+
+    @property
+    def searches(self):
+        return self._L.ddx_stream_searches(self.h)
 
     def in_flight(self):
         return self._L.ddx_stream_in_flight(self.h)

@@ -14,15 +14,17 @@ counters, then stops. Three scores, as tables per second:
           from the launch -- the bench's value; the default
   window  jobs finished in the timed window, a job counting 1/jobs_per_deal of a table; it
           decays as heavy jobs pile up on the lanes, so it favours draining easy jobs
-  launch  jobs finished from the launch to the end of the window, over that time Every answer a candidate finishes is compared with the
-first candidate's answers for the same deals (all candidates are exact solvers; a difference
-is a bug and aborts the sweep).
+  launch  jobs finished from the launch to the end of the window, over that time
+Every answer a candidate finishes is compared with the first candidate's answers for the same
+deals (all candidates are exact solvers; a difference is a bug and aborts the sweep).
 
 Swept: lanes (threads per CU x 256 CUs, with the kernel held to 3 or 4 waves per SIMD where
 the threads need it), lanes per search (one lane, or a 16-lane team), TT_LOG2
 per search (one lane: 9..12, i.e. 0.16-1.3 MB of TT per search and up to 258 GB in all of the
 288 GB; a team: 13..14), jobs per deal (5 = one job per strain, 20 = one per lead) and the stage schedule
-(priority / chain / split, or none: the per-thread kernel). The best is written to `out` under the workload's name; bench.py
+(priority / chain / split, or none: the per-thread kernel). A batch that runs with a wave per
+search (ddx_gpu_waves) depends on the number of searches, TT_LOG2 and the jobs per deal alone:
+candidates that differ in nothing else are measured once. The best is written to `out` under the workload's name; bench.py
 and the tools read the "full" entry.
 """
 import argparse
@@ -75,13 +77,24 @@ def candidates(quick):
     return out
 
 
-def measure(cfg, hands, warmup_s, measure_s):
-    """Sustained tables/s of one candidate; returns (score, answers, details)."""
+def same_run(cfg, waves):
+    """What a candidate's run depends on, given its searches on waves (0: one lane per search)."""
+    return (waves, cfg["tt_log2"], cfg["jobs_per_deal"]) if waves else tuple(sorted(cfg.items()))
+
+
+def measure(cfg, hands, warmup_s, measure_s, measured):
+    """Sustained tables/s of one candidate; returns (score, answers, details), or None when one that
+    runs alike is among `measured`."""
     n = len(hands)
     dev = torch.device("cuda:0")
     d_hands = torch.from_numpy(hands.view(np.int64)).to(dev)
     d_out = torch.empty((n, 20), dtype=torch.uint8, device=dev)
     g = ddx.GpuSolver(graph=True, **cfg)
+    waves = g.waves(n)
+    if same_run(cfg, waves) in measured:
+        g.close()
+        return None
+    measured.add(same_run(cfg, waves))
     torch.cuda.synchronize()
     g.solve_async(d_hands.data_ptr(), n, d_out.data_ptr(), stream=torch.cuda.current_stream().cuda_stream)
     t0 = time.perf_counter()
@@ -100,7 +113,7 @@ def measure(cfg, hands, warmup_s, measure_s):
     window = (j1 - j0) / jpd / (t2 - t1)
     launch = j1 / jpd / (t2 - t0)
     whole = int((out != 255).all(axis=1).sum()) / (t_stop - t0)
-    return window, out, {"whole_tables_per_s": round(whole, 2), "tables_per_s_from_launch": round(launch, 2),
+    return window, out, {"waves": waves, "whole_tables_per_s": round(whole, 2), "tables_per_s_from_launch": round(launch, 2),
                          "nodes_per_s": round((n1 - n0) / (t2 - t1)), "warm_jobs": int(j0),
                          "timed_jobs": int(j1 - j0), "startup_s": round(t1 - t0 - warmup_s, 3)}
 
@@ -122,8 +135,13 @@ def main():
     log("workload %s: %d deals" % (a.workload, len(hands)))
     ref = None
     results = []
+    measured = set()
     for cfg in (json.loads(a.candidates) if a.candidates else candidates(a.quick)):
-        score, out, det = measure(cfg, hands, a.warmup_s, a.measure_s)
+        got = measure(cfg, hands, a.warmup_s, a.measure_s, measured)
+        if got is None:
+            log("as before: %s" % json.dumps(cfg))
+            continue
+        score, out, det = got
         if ref is None:
             ref = out
         both = (out != 255) & (ref != 255)

@@ -240,10 +240,15 @@ int ddx_mlp_load(ddx_mlp* h, const char* path);
 
 /* One persistent kernel fed through `ring_slots` pinned host slots; each deal's table is
  * published as soon as it is solved, in any order. Replaces dd_stream's kernel and ring
- * (gpu/stream_main.cu:38-114, 146-164). cfg->jobs_per_deal 20 keeps more lanes busy than 5
- * when ring_slots * jobs_per_deal is near the lane count. */
+ * (gpu/stream_main.cu:38-114, 146-164). Each search has a wave of its own; only device, lanes / team,
+ * tt_log2, jobs_per_deal and seed_mode matter (the signature-entry and shared-TT builds run one lane
+ * per search, and waves_per_simd 3 matters as well). cfg->jobs_per_deal 20 keeps more searches busy
+ * than 5 when ring_slots * jobs_per_deal is near their number. The net's calls run beside an open
+ * stream; opening another solver or stream on the device waits until it is closed. */
 typedef struct ddx_stream ddx_stream;
 int ddx_stream_open(const ddx_gpu_config* cfg, int ring_slots, ddx_stream** out);
+/* Searches that run at once, each with its own TT: lanes / team, at most 16 per CU. */
+int64_t ddx_stream_searches(const ddx_stream* s);
 /* Queues one deal (hands N,E,S,W; seeds20 = NS-trick seeds [strain][declarer] for the seeded
  * modes, else NULL) under a caller id. Returns DDX_OK, or DDX_E_FULL when every slot is in
  * use (poll, then push again). Safe to call from one producer thread while another polls. */
