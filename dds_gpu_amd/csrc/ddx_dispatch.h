@@ -34,15 +34,26 @@ struct Dispatch {
   long long searches;  // the kernel uses this many of the handle's TTs, stacks and generations
 };
 
-// Batches run with one wave per search, but for those that keep very many lanes busy for long:
-// measured on full deals, 65,536 lanes enter 1.86e9 nodes/s and the wave kernel 3.3e9, but 196,608
-// lanes 3.8e9 while their job queue lasts. A queue shorter than two jobs per lane is mostly tail:
-// 327,680 jobs (8-card endings) on 196,608 lanes take 820 ms with lanes, 380 ms with waves. The
-// measuring options (stage profile, LDS line cache, splitting) exist in the lane kernels only.
-// A handle of at most 1,024 lanes with a long queue (over eight jobs per lane) also stays with
-// the 16 waves that its lanes fill: it is a solver in a corner of the device, and a wave per search
-// would take 64 times as much of it. (The test of stop requests counts on such a batch still
-// running after 1.5 s; the wave kernel would be done with it.)
+// Batches run with one wave per search (ddx_wave.hip), but for three kinds, which stay on lanes.
+//
+// The measuring options (stage profile, LDS line cache, splitting) exist in the lane kernels only.
+//
+// saturated: more than 65,536 lanes with more than two jobs each. Two jobs a lane are where lanes
+// begin to win for full deals under a time limit, the work that such lane counts are tuned for: on
+// 196,608 lanes for 80 s, 100,000 deals (2.5 jobs a lane, TT_LOG2 12) give 53,854 whole tables with
+// lanes and 38,409 with waves, 78,000 deals (2.0, TT_LOG2 11) 42,134 and 33,562, 20,000 deals (0.5,
+// 40 s) 10,048 and 17,769. Lanes start every job early and leave the heavy ones for last. Batches that
+// run to their end are the other way round up to many jobs a lane: eight-card endings 807 ms with
+// lanes and 380 with waves at 1.7 jobs a lane, 827 and 487 at 2.2, 1,150 and 895 at 4.1, 1,800 and 1,746
+// at 8.1; six-card endings 180 and 178 at 4.1, 311 and 354 at 8.1. (65,536 lanes or fewer, two waves per
+// SIMD at most, enter 1.9e9 nodes/s and waves 2.9e9 to 3.3e9.)
+//
+// corner: at most 1,024 lanes with more than eight jobs each. Nothing but time speaks for lanes here:
+// 3,000 ten-card deals on 1,024 lanes take 16.4 s, and 0.80 s with waves; 1,700 eight-card ones 1.33 s
+// and 44 ms. (Beside it another batch of 351 ms takes 355-378 ms all that time, or 405 ms once.) Such a
+// handle's long batches run as they always have, on the 16 waves that its lanes fill, because the test
+// of stop requests (tests/test_gpu.py) takes it that the former batch still runs after 1.5 s. With team 16
+// and 16 times the lanes, the same number of searches runs on waves.
 //
 // wave_cap: waves of the wave kernel that the device holds at once; 0 in builds without it.
 inline Dispatch dispatch(const ddx_gpu_config& c, int wave_cap, long long jobs) {

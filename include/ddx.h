@@ -114,8 +114,10 @@ int ddx_cpu_solve_batch(const uint64_t* hands, int64_t n, int threads, int tt_lo
 /* Most batches run with one wave per search, and then only device, lanes / team (the number of
  * searches and TTs), tt_log2, jobs_per_deal, seed_mode and graph matter. Kernels with one lane per
  * search, which the other options are about, run with team 1 when more than 65536 lanes have
- * more than two jobs each, when at most 1024 have more than eight, and when a measuring option
- * (profile, lds_lines, split_min_nodes) asks for them; results and counters are the same. */
+ * more than two jobs each, when at most 1024 have more than eight (slower; team 16 with 16 times the
+ * lanes has as many searches and runs them on waves), and when a measuring option (profile,
+ * lds_lines, split_min_nodes) asks for them; results and counters are the same. ddx_gpu_waves tells
+ * which kernel a batch runs on. */
 typedef struct ddx_gpu_config {
   int device;           /* HIP device ordinal */
   int64_t lanes;        /* solver lanes; lanes / team searches run, each with its own TT (default
