@@ -951,7 +951,7 @@ static void sync_bf16(ddx_mlp* h) {
 // Seeds of n deals on stream s. Few deals are spread over a block per sample tile; from 512 deals
 // (640 blocks) on, the persistent kernel is faster although its blocks have less than a group of
 // 16 deals per CU then. Beside a stream, and in a capture, whose replays may be beside one, any
-// number of deals goes tile by tile: 100,000 deals in 2.1 ms beside a stream, 0.41 ms otherwise.
+// number of deals goes tile by tile: 100,000 deals in 2.1 ms beside a stream, 0.39 ms otherwise.
 static void launch_predict(const ddx_mlp* h, hipStream_t s, const uint64_t* d_hands, long long n, uint8_t* d_seeds,
                            bool captured) {
   const long long groups = (n + 15) / 16;

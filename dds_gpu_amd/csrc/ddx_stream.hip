@@ -51,8 +51,9 @@ __device__ __forceinline__ int load_relaxed_sys(int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// One lane per search, for the builds without a wave-per-search kernel (ddx_stream_wave.hip). Values the host changes while the kernel runs (produced, eof, stop) live in host memory: one lane of the wave reads them,
-// at most every DDX_STREAM_POLL rounds and only while some lane waits for input, and
+// One lane per search, for the builds without a wave-per-search kernel (ddx_stream_wave.hip). Values
+// the host changes while the kernel runs (produced, eof, stop) live in host memory: one lane of the
+// wave reads them, at most every DDX_STREAM_POLL rounds and only while some lane waits for input, and
 // broadcasts them to the wave. The reads are relaxed; only when they show something new (more
 // deals, the end) does that lane add the system-scope acquire that makes the host's slot
 // contents visible. An acquire at system scope invalidates the caches the whole GPU shares,
@@ -244,10 +245,9 @@ extern "C" int ddx_stream_open(const ddx_gpu_config* cfg_in, int ring_slots, ddx
   s->ring = ring_slots;
   s->work_ring = 1;
   while (s->work_ring < 4 * s->ring) s->work_ring <<= 1;
-  // One wave per search (ddx_stream_wave.hip), in the builds that have it: 1,500 eight-card deals
-  // through 4,096 searches and a ring of 256 took 912 ms with one lane per search, 45 ms now. TTs only
-  // for the searches that run: more would lie unused, and memory that others freed has to be
-  // cleared by the driver first (10 GB took 250 ms).
+  // One wave per search (ddx_stream_wave.hip), in the builds that have it. TTs only for the searches
+  // that run: more would lie unused, and memory that others freed has to be cleared by the driver
+  // first (10 GB took 250 ms).
   StreamGrid waves;
   int rc = stream_wave_grid(cfg.device, cfg.lanes / cfg.team, &waves);
   if (rc != DDX_OK) {

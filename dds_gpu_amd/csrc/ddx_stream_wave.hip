@@ -3,8 +3,10 @@
 //
 // A deal's latency is its slowest lead's, and a lead's speed is its search's: a search on a wave
 // runs at 1.15M nodes/s alone, as in a batch, where a 16-lane team ran at 115k under full load and
-// one lane at 20-150k. 1,500 eight-card deals through a ring of 256 slots: 891 ms with one lane per
-// search, 44 ms with waves.
+// one lane at 20-150k. 1,500 eight-card deals through a ring of 256 slots: 1,011 ms with one lane per
+// search, 52 ms with waves; 40,000 of them in a ring that holds all 932 and 283 ms, although 196,608
+// lanes then stand against 4,096 waves. (80 VGPRs: 87 scalar registers are spilled to vector lanes, 12
+// vector registers to scratch.)
 //
 // The ring is ddx_stream.hip's. Reading the host's counters costs a PCIe round trip, so only the
 // first kPollers waves do it, whether idle or between the nodes of a search, and publish what they

@@ -9,17 +9,18 @@
 // parallel (ddx_wave.hpp). Measured: one search alone 1.15M nodes/s (nine-card endings); with
 // every wave slot filled 2.9e9 nodes/s on eight-card endings, 3.3e9 on full deals -- above the
 // lane kernel's 1.9e9 with 65,536 lanes, below its 3.8e9 with 196,608 lanes held to three waves
-// per SIMD while its job queue lasts. 256 seven-card endings on 1,280 searches: 174 ms with lanes,
-// 7.4 ms here; 500 nine-card endings 1,396 -> 90 ms; 65,536 eight-card endings on 196,608
-// searches 820 -> 380 ms.
+// per SIMD while its job queue lasts. 256 seven-card endings on 1,280 searches: 157 ms with lanes,
+// 8.4 ms here; 500 nine-card endings 1,602 -> 96 ms; 65,536 eight-card endings on 196,608
+// searches 829 -> 385 ms. (Times of random batches, both ways on the same deals; their heaviest jobs
+// make batches of other deals differ by a quarter.)
 //
 // With every slot filled the kernel is bound by the scalar unit (one instruction per four cycles
 // and SIMD: 181 scalar, 114 vector instructions and 22 jumps per node, the scalar ones 85% of the
 // time). Alone, a node's 330 instructions take four cycles each and it waits half as long again:
 // for jumps (38 cycles when taken), the TT and the way between the vector and the scalar unit. Six
-// waves per SIMD (80 VGPRs; scalar registers spilled to vector lanes): 5 and 6 measure 390 and
-// 380 ms on 65,536 eight-card endings (and one search alone the same within 1%); 4 were 6% slower
-// than 6, and 8 spill vector registers and cost one search 7%.
+// waves per SIMD (80 VGPRs; 83 scalar registers spilled to vector lanes, 5 vector registers to
+// scratch): 5 and 6 measure 390 and 380 ms on 65,536 eight-card endings (and one search alone the same within 1%); 4 were 6% slower
+// than 6, and 8 spill many more vector registers and cost one search 7%.
 #include <hip/hip_runtime.h>
 
 #include "ddx_wave.h"
