@@ -32,6 +32,8 @@ enum class BatchKernel {
 struct Dispatch {
   BatchKernel kernel;
   long long searches;  // the kernel uses this many of the handle's TTs, stacks and generations
+  int waves_per_simd;  // lane kernels: 0, 3 or 4 (beside a stream never the compiler's own 230 to 260 VGPRs
+                       // where there is a kernel held to 168)
 };
 
 // Batches run with one wave per search (ddx_wave.hip), but for three kinds, which stay on lanes.
@@ -55,22 +57,27 @@ struct Dispatch {
 // of stop requests (tests/test_gpu.py) takes it that the former batch still runs after 1.5 s. With team 16
 // and 16 times the lanes, the same number of searches runs on waves.
 //
-// wave_cap: waves of the wave kernel that the device holds at once; 0 in builds without it.
-inline Dispatch dispatch(const ddx_gpu_config& c, int wave_cap, long long jobs) {
-  if (jobs <= 0) return {BatchKernel::kNone, 0};
+// Beside an open stream both of these rules are off: most lane kernels need more registers than the
+// stream leaves (kRoomVgprs below), and would wait until it is closed.
+//
+// wave_cap: waves of the wave kernel that the device holds at once; 0 in builds without it. beside:
+// a stream is open on the device.
+inline Dispatch dispatch(const ddx_gpu_config& c, int wave_cap, long long jobs, bool beside) {
+  if (jobs <= 0) return {BatchKernel::kNone, 0, 0};
   const bool measuring = c.profile || c.lds_lines || c.split_min_nodes > 0;
   const bool saturated = c.team == 1 && c.lanes > 65536 && jobs > 2 * c.lanes;
   const bool corner = c.team == 1 && c.lanes <= 1024 && jobs > 8 * c.lanes;
-  if (wave_cap > 0 && !measuring && !saturated && !corner) {
+  if (wave_cap > 0 && !measuring && (beside || (!saturated && !corner))) {
     long long s = c.lanes / c.team;
     if (s > wave_cap) s = wave_cap;
-    return {BatchKernel::kWave, s < jobs ? s : jobs};
+    return {BatchKernel::kWave, s < jobs ? s : jobs, 0};
   }
-  if (c.split_min_nodes > 0) return {BatchKernel::kSplit, c.lanes};
-  if (c.lds_lines) return {BatchKernel::kLds, c.lanes};
-  if (c.waves_per_simd) return {BatchKernel::kHeld, c.lanes};
+  const int w = beside && !c.waves_per_simd ? 3 : c.waves_per_simd;
+  if (c.split_min_nodes > 0) return {BatchKernel::kSplit, c.lanes, w};
+  if (c.lds_lines) return {BatchKernel::kLds, c.lanes, w};
+  if (c.waves_per_simd) return {BatchKernel::kHeld, c.lanes, w};
   // Teams have a lane kernel only for the stage profile.
-  return {BatchKernel::kSchedule, c.profile ? c.lanes / c.team : c.lanes};
+  return {BatchKernel::kSchedule, c.profile ? c.lanes / c.team : c.lanes, 0};
 }
 
 // The wave-per-search stream kernel stays on the device until the stream is closed, and the net's

@@ -116,8 +116,10 @@ int ddx_cpu_solve_batch(const uint64_t* hands, int64_t n, int threads, int tt_lo
  * search, which the other options are about, run with team 1 when more than 65536 lanes have
  * more than two jobs each, when at most 1024 have more than eight (slower; team 16 with 16 times the
  * lanes has as many searches and runs them on waves), and when a measuring option (profile,
- * lds_lines, split_min_nodes) asks for them; results and counters are the same. ddx_gpu_waves tells
- * which kernel a batch runs on. */
+ * lds_lines, split_min_nodes) asks for them; results and counters are the same. Beside an open
+ * stream only the measuring options run lane kernels, which there are held to 3 waves per SIMD; those
+ * of the stage profile wait until the stream is closed. ddx_gpu_waves tells which kernel a batch runs
+ * on. */
 typedef struct ddx_gpu_config {
   int device;           /* HIP device ordinal */
   int64_t lanes;        /* solver lanes; lanes / team searches run, each with its own TT (default
@@ -165,8 +167,8 @@ int ddx_gpu_open(const ddx_gpu_config* cfg, ddx_gpu** out);
 void ddx_gpu_close(ddx_gpu* h);
 /* Device bytes held by the handle. */
 uint64_t ddx_gpu_device_bytes(const ddx_gpu* h);
-/* Searches that a batch of n deals runs with, each on a wave of its own; 0 when a kernel with one
- * lane per search runs it (see above). */
+/* Searches that a batch of n deals would run with now, each on a wave of its own; 0 when a kernel
+ * with one lane per search would run it (see above). */
 int64_t ddx_gpu_waves(const ddx_gpu* h, int64_t n);
 
 /* Solves n deals: host hands[4n] in, host out[20n] (0xFF = unsolved after a stop). seeds:
@@ -245,8 +247,10 @@ int ddx_mlp_load(ddx_mlp* h, const char* path);
  * (gpu/stream_main.cu:38-114, 146-164). Each search has a wave of its own; only device, lanes / team,
  * tt_log2, jobs_per_deal and seed_mode matter (the signature-entry and shared-TT builds run one lane
  * per search, and waves_per_simd 3 matters as well). cfg->jobs_per_deal 20 keeps more searches busy
- * than 5 when ring_slots * jobs_per_deal is near their number. The net's calls run beside an open
- * stream; opening another solver or stream on the device waits until it is closed. */
+ * than 5 when ring_slots * jobs_per_deal is near their number. Its kernel stays on the device until
+ * it is closed. The net's calls and batches of open handles run beside it; opening another solver
+ * or stream on the device waits, and so do kernels of other libraries that need more registers than
+ * it leaves: 192 VGPRs per SIMD with 16 searches per CU or more, 352 with 8. */
 typedef struct ddx_stream ddx_stream;
 int ddx_stream_open(const ddx_gpu_config* cfg, int ring_slots, ddx_stream** out);
 /* Searches that run at once, each with its own TT: lanes / team, at most 16 per CU. */

@@ -25,15 +25,20 @@ int main() {
                     ddx_gpu_config c{0, L, 10, jpd, schedule, 0, block, profile, team, 0, waves, lds, split};
                     if (!gpu_config_ok(c, 9, 20)) continue;
                     configs++;
-                    for (int cap : {0, 6144}) {
+                    for (int mode = 0; mode < 4; mode++) {
+                      const int cap = mode & 1 ? 6144 : 0;
+                      const bool beside = mode & 2;
                       if (cap == 0 && team != 1) continue;  // the builds without wave kernels have no teams
                       for (long long n : {0ll, 1ll, 12ll, 13ll, 409ll, 410ll, 2000ll, 13107ll, 26215ll, 100000ll}) {
-                        const Dispatch d = dispatch(c, cap, n * jpd);
+                        const Dispatch d = dispatch(c, cap, n * jpd, beside);
                         batches++;
                         const bool none = d.kernel == BatchKernel::kNone, wave = d.kernel == BatchKernel::kWave;
                         if (d.searches > L / team || none != (n == 0) || none != (d.searches == 0)) bad++;
                         if (wave && (d.searches > cap || d.searches > n * jpd || profile || lds || split)) bad++;
                         if (!wave && !none && d.searches != (profile ? L / team : L)) bad++;  // the lane kernels' grids
+                        // Beside a stream: waves, or a lane kernel held to 168 or 128 VGPRs, but for the profile.
+                        if (beside && cap && !none && !wave && !profile && d.waves_per_simd < 3) bad++;
+                        if (!beside && !none && !wave && d.waves_per_simd != waves) bad++;
                       }
                     }
                   }

@@ -110,8 +110,22 @@ def batch_case(ddx):
             assert np.array_equal(out, want) and st.nodes == cpu.nodes
 
 
+def lanes_case(ddx):
+    """Batches that run with one lane per search go to waves, or to a kernel held to 3 waves per SIMD."""
+    hands = ddx.random_deals(33, 6600, 5)
+    want, cpu = ddx.cpu_solve(hands, threads=8, tt_log2=9, jobs_per_deal=20)
+    for kw, waves in ((dict(lanes=65792), 6144), (dict(lanes=65792, graph=True), 6144), (dict(lanes=16384, lds_lines=3), 0),
+                      (dict(lanes=1024), 1024)):
+        with ddx.GpuSolver(tt_log2=9, jobs_per_deal=20, schedule=ddx.SCHED_SPLIT, **kw) as g:
+            def solve():
+                out, st = timed("%s, on %d waves" % (kw, g.waves(len(hands))), lambda: g.solve(hands))
+                assert np.array_equal(out, want) and st.nodes == cpu.nodes and st.tt_stores == cpu.tt_stores
+                return g.waves(len(hands))
+            assert (solve(), beside_stream(ddx, solve), solve()) == (0, waves, 0)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", ["net", "growth", "batch"])
+@pytest.mark.parametrize("case", ["net", "growth", "batch", "lanes"])
 def test_runs_while_a_stream_is_open(case):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), case], cwd=ROOT, capture_output=True, text=True,
                        timeout=100)
@@ -162,4 +176,4 @@ if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     import torch  # noqa: F401 -- before the ddx library: one HIP runtime for both
     from dds_gpu_amd import ddx as module
-    {"net": net_case, "growth": growth_case, "batch": batch_case}[sys.argv[1]](module)
+    {"net": net_case, "growth": growth_case, "batch": batch_case, "lanes": lanes_case}[sys.argv[1]](module)
