@@ -50,8 +50,8 @@ struct Dispatch {
 // at 8.1; six-card endings 180 and 178 at 4.1, 311 and 354 at 8.1. (65,536 lanes or fewer, two waves per
 // SIMD at most, enter 1.9e9 nodes/s and waves 2.9e9 to 3.3e9.)
 //
-// corner: at most 1,024 lanes with more than eight jobs each. Nothing but time speaks for lanes here:
-// 3,000 ten-card deals on 1,024 lanes take 16.4 s, and 0.80 s with waves; 1,700 eight-card ones 1.33 s
+// corner: at most 1,024 lanes with more than eight jobs each. No figure speaks for lanes here: 3,000
+// ten-card deals on 1,024 lanes take 16.4 s, and 0.80 s with waves; 1,700 eight-card ones 1.33 s
 // and 44 ms. (Beside it another batch of 351 ms takes 355-378 ms all that time, or 405 ms once.) Such a
 // handle's long batches run as they always have, on the 16 waves that its lanes fill, because the test
 // of stop requests (tests/test_gpu.py) takes it that the former batch still runs after 1.5 s. With team 16
